@@ -28,7 +28,7 @@ using mr::MlpView;
 // activations, 512 a row. The tile's h1 and h2 pass through LDS; the four
 // wavefronts take turns at the small output layer. Two workgroups share a CU, one
 // in its products while the other evaluates GELU.
-// Measured, 100,003 rows: 160 -> 63 us; 8192 rows with trace: 48 -> 19 us.
+// Measured, 100,003 rows: 160 -> 84 us; 8192 rows with trace: 48 -> 21 us.
 constexpr uint32_t kForwardGroups = 512u;  // two per CU
 
 template <bool kTrace>
@@ -166,7 +166,7 @@ extern "C" __global__ void __launch_bounds__(256) mr_mlp_sum_kernel(const float*
 // laid out like the forward kernel: each of four wavefronts holds its 64 columns
 // of W2 (now by input) in registers, dz2 of the tile goes to memory in FP32 and
 // to LDS as the BF16 operand of the second product.
-// Measured, 8192 rows: 6.7 + 69 us (elementwise pass, strided GEMM) -> 22 us.
+// Measured, 8192 rows: 6.7 + 69 us (elementwise pass, strided GEMM) -> 25 us.
 __global__ void __launch_bounds__(256, 2) mlp_hidden_backward_kernel(MlpView m, const float* dy, const float* z2,
                                                                      const float* z1, uint32_t n, float* dz2,
                                                                      float* dz1) {
