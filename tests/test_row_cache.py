@@ -12,14 +12,19 @@ import oracle_lib as ol
 BOX, PLANE = 2, 3
 
 
-def flat_chain(boxes):
-    """A floating chain of box links lying on a plane: four contacts a link."""
-    links = [mu.body(2.0, [0.02] * 3)]
+def flat_chain(boxes, mass=None):
+    """A floating chain of box links lying on a plane: four contacts a link. `mass(i)` replaces link i's mass."""
+    def link(i, m, inertia, **joint):
+        if mass is not None:
+            m, inertia = mass(i), [mass(i) * x for x in (0.01, 0.012, 0.014)]
+        return mu.body(m, inertia, **joint)
+
+    links = [link(0, 2.0, [0.02] * 3)]
     shapes = [mu.shape(0, BOX, (0.1, 0.1, 0.05))]
     dofs = [mu.dof(0, mu.INVALID) for _ in range(6)]
     for i in range(1, boxes):
-        links.append(mu.body(1.0 + 0.1 * i, [0.01, 0.012, 0.014], parent=i - 1, joint_type=0, q_index=6 + i,
-                             v_index=5 + i, axis=(0, 1, 0), parent_anchor=(0.12, 0, 0), child_anchor=(-0.12, 0, 0)))
+        links.append(link(i, 1.0 + 0.1 * i, [0.01, 0.012, 0.014], parent=i - 1, joint_type=0, q_index=6 + i,
+                          v_index=5 + i, axis=(0, 1, 0), parent_anchor=(0.12, 0, 0), child_anchor=(-0.12, 0, 0)))
         dofs.append(mu.dof(i, 6 + i, drive=(0, 0, 0.02, 0)))
         shapes.append(mu.shape(i, BOX, (0.1, 0.1, 0.05)))
     ground = mu.body(0.0, [1, 1, 1], motion=0)
@@ -54,3 +59,33 @@ def test_rows_in_lds_and_in_global_memory_match_oracle(gpu, boxes, tolerance):
         gq, gv, _ = world.state()
         assert np.array_equal(gq.view(np.uint32), ost.q.view(np.uint32)), k
         assert np.array_equal(gv.view(np.uint32), ost.v.view(np.uint32)), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heavy,fails_at", [(1, 5), (3, 13), (14, 57)])
+def test_a_non_finite_update_reports_its_contact_in_lds_and_in_global_memory(gpu, heavy, fails_at):
+    """A chain of light boxes and a heavy one falls at 1e37 m/s: an impulse of the heavy box overflows in
+    the first sweep, at a contact whose record is in LDS (about the first nine are) or behind them. The
+    oracle counts sweeps and takes residuals only after they all passed."""
+    boxes = 16
+    w = flat_chain(boxes, lambda i: 100.0 if i == heavy else 0.2)
+    cfg = w.config(pair_capacity=128, manifold_capacity=64, constraint_capacity=96)
+    world, ost = mr.World(w.model, cfg), ol.OracleState(w.model, cfg)
+    q, v = np.zeros((w.envs, w.nq), np.float32), np.zeros((w.envs, w.nv), np.float32)
+    q[:, 2], q[:, 6], v[:, 2] = 0.0495, 1.0, -1.0e37
+    scene = np.zeros((w.envs, 1), mr.BODY_STATE_DTYPE)
+    scene[:] = mu.scene_state((0, 0, 0), motion=0)
+    ost.q[:], ost.v[:], ost.scene[:] = q, v, scene
+    world.set_state(q, v, scene)
+    cmd = np.zeros((w.envs, w.nv), np.float32)
+    status, cs = ost.step(cmd, control_step=0)[:2]
+    assert np.all(status["code"] != 0) and np.all(status["failing_index"] == fails_at), status["failing_index"]
+    assert np.all(cs["solver_iterations"] == 0) and np.all(cs["constraints"] == 4 * boxes)
+    world.advance(cmd[None])
+    got = world.statuses()[0]
+    for f in ("code", "failing_index", "successful_substeps"):
+        np.testing.assert_array_equal(got[f], status[f], err_msg=f)
+    np.testing.assert_array_equal(world.contact_statuses()[0]["constraints"], cs["constraints"])
+    gq, gv, _ = world.state()
+    assert np.array_equal(gq.view(np.uint32), ost.q.view(np.uint32))
+    assert np.array_equal(gv.view(np.uint32), ost.v.view(np.uint32))
