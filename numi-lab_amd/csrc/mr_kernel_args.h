@@ -157,11 +157,11 @@ struct LdsLayout {
     uint32_t rslot;  // [slots][6][64] floats: outward spatial accelerations
     uint32_t rstack; // [stack][64] floats: joint terms of the inward path
     uint32_t resid;  // [2][constraint_capacity] floats (+ 1): per-constraint residual terms (after responses);
-                     // before them the contact schedule's levels
-    uint32_t sbody;  // [max_scene_bodies][5] float4: solver bodies of the ordered sweeps (after responses)
-    uint32_t sord;   // [constraint_capacity] u16: contacts in schedule order (after responses)
-    uint32_t rows;       // floats to the end of the layout: cached rows and blocks of the unscheduled sweeps,
-    uint32_t rows_words; // over sbody and sord (the scheduled ones' arrays); 0 with the Jacobi solver
+                     // before them the contact schedule's level words
+    uint32_t sord;   // [2][constraint_capacity] u16 behind those words: contacts in schedule order, their levels
+    uint32_t sbody;  // [max_scene_bodies][5] float4 over the levels: solver bodies of the ordered sweeps
+    uint32_t rows;       // floats from the second residual array to the layout's end: cached rows and blocks
+    uint32_t rows_words; // of the unscheduled sweeps, read before that array is written; 0 with Jacobi
     uint32_t jrelax; // [constraint_capacity] floats: relaxed-Jacobi damping per contact (after responses)
     uint32_t jdelta; // [constraint_capacity][3] floats: relaxed-Jacobi impulse deltas (after responses)
     // MLP instance of the kernel only (past the plain layout's end):
@@ -243,6 +243,7 @@ struct KernelArgs {
 
 // LDS bytes of one warm-start MLP tile: 16 x 8 FP32 inputs and two
 // 16 x 264 BF16 hidden layers.
+constexpr uint32_t kMaxConstraints = 4096u;  // largest constraint_capacity
 constexpr uint32_t kMlpTileLdsBytes = 16u * 8u * 4u + 2u * 16u * 264u * 2u;
 // One captured sample: 8 features, the converged impulse (3), a valid flag,
 // the warm start the cone solve began from (3), 1.0 where the network

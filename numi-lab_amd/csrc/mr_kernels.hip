@@ -3205,13 +3205,18 @@ MRD_INL void solver_apply_impulse(float4* b, V3 x, V3 imp) {
 }
 
 // Builds the schedule: e.sord gets the contacts between scene bodies sorted by level (index order
-// within one), then the articulated contacts in index order; the second half of e.resid gets one
-// word per level and one behind the last: the level's first entry in e.sord | (its articulated
-// contact + 1) << 16. Returns the number of levels; the total of the last word is the number of
-// contacts between scene bodies. Needs nscene < 64 (MR_MAX_BODIES counts the links too).
+// within one), then the articulated contacts in index order; e.resid gets one word per level and
+// one behind the last: the level's first entry in e.sord | (its articulated contact + 1) << 16.
+// Returns the number of levels; the total of the last word is the number of contacts between
+// scene bodies. Needs nscene < 64 (MR_MAX_BODIES counts the links too).
+//
+// The schedule takes no LDS of its own at a large contact capacity c: its 4 (c + 1) bytes of level
+// words, 2 c of order and, while it is built, 2 c of the contacts' levels lie in the residual
+// arrays' 8 c + 4, which are written when it is no longer read (the first half with the last
+// sweep done, the second after the pass that still reads e.sord).
 MRD_INL uint32_t schedule_contacts(const Env& e, uint32_t lane, uint32_t ncons, uint32_t ccap) {
-    uint32_t* lev = reinterpret_cast<uint32_t*>(e.resid);
-    uint32_t* pack = lev + ccap;
+    uint32_t* pack = reinterpret_cast<uint32_t*>(e.resid);
+    uint16_t* lev = e.sord + ccap;
     uint32_t body_level = 0u;  // lane s: the first level scene body s is free at
     uint32_t art_level = 0u, levels = 0u;
     for (uint32_t base = 0; base < ncons; base += kLanes) {
@@ -3233,7 +3238,7 @@ MRD_INL uint32_t schedule_contacts(const Env& e, uint32_t lane, uint32_t ncons, 
             body_level = ((da && lane == a) || (db && lane == b)) ? l : body_level;
             levels = levels > l ? levels : l;
         }
-        if (lane < n) lev[base + lane] = mine;
+        if (lane < n) lev[base + lane] = (uint16_t)mine;
     }
     __syncthreads();
     uint32_t at = 0u;
@@ -3397,6 +3402,7 @@ struct StageClock {
 // ------------------------------------------------ learned warm start
 
 static_assert(mr::kMlpTileLdsBytes == mr::kMlpLdsBytes, "MLP tile LDS size");
+static_assert(mr::kMlpTileLdsBytes >= 4u * mr::kMaxConstraints, "a second attempt's residual terms fit the MLP tile");
 // Normalized features beyond this many training standard deviations keep the
 // plain warm start.
 constexpr float kMlpFeatureBound = 8.0f;
@@ -4323,7 +4329,7 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
         uint32_t levels = 0u, nart = ncons;
         if (scheduled) {
             levels = schedule_contacts(e, lane, ncons, ccap);
-            nart = ncons - uniform_u32(reinterpret_cast<const uint32_t*>(e.resid)[ccap + levels]);
+            nart = ncons - uniform_u32(reinterpret_cast<const uint32_t*>(e.resid)[levels]);
         }
         // articulated contact k of the substep: the k-th in index order (the
         // Jacobi mode keeps no list: its loops pass the others by)
@@ -4634,7 +4640,7 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
             // DoF lanes accumulate the warm-start impulses of the articulated
             // contacts in index order, the next contact's response rows in flight;
             // scene bodies take theirs in schedule order.
-            const uint32_t* pack = reinterpret_cast<const uint32_t*>(e.resid) + ccap;
+            const uint32_t* pack = reinterpret_cast<const uint32_t*>(e.resid);
             const uint32_t pack_lane = scheduled && lane <= levels ? pack[lane] : 0u;
             auto level_pack = [&](uint32_t l) { return l < kLanes ? read_lane(pack_lane, l) : uniform_u32(pack[l]); };
             // the scene contact of this lane in a level of n entries from `first`
@@ -4922,8 +4928,10 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
                     if (!missed && A.mlp.max_normal_residual > 0.0f) {
                         // The learned solve reached the tolerance: its normal
                         // residuals, computed as the residual pass below does,
-                        // must also stay within max_normal_residual.
-                        float* res_n = e.resid;
+                        // must also stay within max_normal_residual. (Their
+                        // articulated terms go to the MLP tile's LDS, free by
+                        // now: a second attempt reads the schedule in e.resid.)
+                        float* res_n = reinterpret_cast<float*>(e.mlp_lds);
                         for (uint32_t c = 0; c < ncons; ++c) {
                             if ((uniform_u32(e.cpair[c] >> 16) & mr::kHotArticulated) == 0u) continue;
                             const float j0 = e.jrow[(size_t)c * 3u * mnv + row_lane()];

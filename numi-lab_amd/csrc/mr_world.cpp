@@ -76,7 +76,7 @@ World::World(const ModelData& model, const MRWorldStepConfigC& config) : model_(
     if (cfg_.pair_capacity == 0u || cfg_.pair_capacity > 4096u) throw std::runtime_error("pair_capacity in [1, 4096]");
     if (cfg_.manifold_capacity == 0u || cfg_.manifold_capacity > 4096u)
         throw std::runtime_error("manifold_capacity in [1, 4096]");
-    if (cfg_.constraint_capacity == 0u || cfg_.constraint_capacity > 4096u)
+    if (cfg_.constraint_capacity == 0u || cfg_.constraint_capacity > kMaxConstraints)
         throw std::runtime_error("constraint_capacity in [1, 4096]");
     if (cfg_.capture_evidence != 0u && cfg_.capture_substep >= cfg_.physics_substeps)
         throw std::runtime_error("capture_substep must be below physics_substeps");
@@ -289,9 +289,13 @@ void World::compute_lds_layout() {
     off = union_start;
     L.resid = take(8u * cfg_.constraint_capacity + 4u, 4u);
     const bool jacobi = cfg_.solver == MR_SOLVER_RELAXED_JACOBI;
-    L.rows = off;
-    L.sbody = take(jacobi ? 0u : 80u * nscene, 16u);
-    L.sord = take(jacobi ? 0u : 2u * cfg_.constraint_capacity, 4u);
+    // The ordered sweeps' schedule (schedule_contacts) lies in the residual arrays: level words,
+    // order, and the solver bodies over the contacts' levels, which only its making reads. The
+    // unscheduled sweeps' record cache starts at the second residual array.
+    L.rows = L.resid + 4u * cfg_.constraint_capacity;
+    L.sord = L.resid + 4u * (cfg_.constraint_capacity + 1u);
+    L.sbody = (L.sord + 2u * cfg_.constraint_capacity + 15u) / 16u * 16u;
+    if (!jacobi) off = std::max(off, L.sbody + 80u * nscene);
     L.jrelax = take(jacobi ? 4u * cfg_.constraint_capacity : 0u, 4u);
     L.jdelta = take(jacobi ? 12u * cfg_.constraint_capacity : 0u, 4u);
     off = std::max(union_end, off);
