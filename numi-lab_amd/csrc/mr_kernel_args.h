@@ -149,7 +149,7 @@ struct LdsLayout {
     uint32_t q, v, vcand, effort, accel, cmd;
     uint32_t pos, rot, w, vl, sa, sl, ca, cl, r;
     uint32_t I, p, Ut, Ub, D, u, L;
-    uint32_t scene, col, ccol, active, npts, moff, okey;
+    uint32_t scene, col, ccol, swept, active, npts, moff, okey;
     uint32_t hfitem, hfq;  // heightfield query table (kHfSlots entries each), collision phase only
     uint32_t lam;    // [constraint_capacity][3] floats: cone impulses
     uint32_t cpair;  // [constraint_capacity]: body_a | body_b << 8 | kind << 16
@@ -244,6 +244,9 @@ struct KernelArgs {
 // LDS bytes of one warm-start MLP tile: 16 x 8 FP32 inputs and two
 // 16 x 264 BF16 hidden layers.
 constexpr uint32_t kMaxConstraints = 4096u;  // largest constraint_capacity
+// LDS that a control-step kernel declares itself, beside the layout above (which a kernel's
+// metadata states too: group_segment_fixed_size 160 in every instance).
+constexpr uint32_t kStepStaticLdsBytes = 160u;
 constexpr uint32_t kMlpTileLdsBytes = 16u * 8u * 4u + 2u * 16u * 264u * 2u;
 // One captured sample: 8 features, the converged impulse (3), a valid flag,
 // the warm start the cone solve began from (3), 1.0 where the network

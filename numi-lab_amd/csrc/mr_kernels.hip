@@ -132,6 +132,7 @@ struct Env {
     float *D, *u, *L;
     MRBodyStateC* scene;
     Collider *col, *ccol;  // ccol: swept colliders of the time-of-impact queries
+    uint32_t* swept;       // [2 kLanes]: pairs waiting for their time-of-impact query
     uint32_t *active, *npts, *moff, *okey;
     uint32_t* hfitem;  // [kHfSlots]: active pair | query << 16
     mr::HfHit* hfq;    // [kHfSlots]: heightfield query results
@@ -3561,6 +3562,9 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
     __shared__ float s_root[7];
     __shared__ MRContactStatusC s_cs;
     __shared__ unsigned long long s_t0;  // start of this control step on the constant-rate clock (step timing)
+    // with the queue instances' next entry; the world's capacities are checked against what is left
+    static_assert(sizeof(s_fail) + sizeof(s_fmax) + sizeof(s_root) + sizeof(s_cs) + sizeof(s_t0) + sizeof(uint32_t) <=
+                      mr::kStepStaticLdsBytes, "static LDS of a control step");
 
     uint32_t lane = stage_lane(threadIdx.x);
     if (env >= args.environment_count) return;
@@ -3616,7 +3620,10 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
     e.L = lds_at<float>(lds_base, L.L);
     e.scene = lds_at<MRBodyStateC>(lds_base, L.scene);
     e.col = lds_at<Collider>(lds_base, L.col);
-    if constexpr (kCcd) e.ccol = lds_at<Collider>(lds_base, L.ccol);
+    if constexpr (kCcd) {
+        e.ccol = lds_at<Collider>(lds_base, L.ccol);
+        e.swept = lds_at<uint32_t>(lds_base, L.swept);
+    }
     e.active = lds_at<uint32_t>(lds_base, L.active);
     e.npts = lds_at<uint32_t>(lds_base, L.npts);
     e.moff = lds_at<uint32_t>(lds_base, L.moff);
@@ -3791,7 +3798,6 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
             // the pairs that overlap, which are few, packed to 64 at a time.
             // With the bounds and the query of each pair in one pass, 372 pairs
             // took 250,000 cycles a segment; 90,000 now (chain of 7 links, 20 boxes).
-            __shared__ uint32_t s_swept[2u * kLanes];
             for (uint32_t s = lane; s < e.nshapes; s += kLanes) {
                 Collider c;
                 ccd_sweep_collider<kGeo>(e, s, remaining, c);
@@ -3804,12 +3810,12 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
                 more = base + kLanes < e.npairs ? 1u : 0u;
                 const bool swept = base + lane < e.npairs && ccd_pair_swept(e, base + lane);
                 const unsigned long long bal = __ballot(swept);
-                if (swept) s_swept[waiting + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = base + lane;
+                if (swept) e.swept[waiting + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = base + lane;
                 waiting = uniform_u32(waiting + (uint32_t)__popcll(bal));
                 __syncthreads();
                 while (waiting >= kLanes || (more == 0u && waiting > 0u)) {
                     if (lane < waiting) {
-                        const uint32_t k = s_swept[lane];
+                        const uint32_t k = e.swept[lane];
                         float toi = 0.0f;
                         const uint32_t r = ccd_pair<kGeo>(e, k, remaining, toi);
                         if (r == kCcdImpact) {
@@ -3823,9 +3829,9 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
                         }
                     }
                     waiting -= waiting < kLanes ? waiting : kLanes;
-                    const uint32_t next = s_swept[kLanes + lane];
+                    const uint32_t next = e.swept[kLanes + lane];
                     __syncthreads();
-                    s_swept[lane] = next;
+                    e.swept[lane] = next;
                     __syncthreads();
                 }
             }

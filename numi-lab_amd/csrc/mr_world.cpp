@@ -24,7 +24,8 @@ hipError_t clock_us_per_tick(float* out);
 
 namespace {
 constexpr uint32_t kColliderBytes = 124u;
-constexpr uint32_t kMaxLdsBytes = 160u * 1024u;
+// dynamic LDS a workgroup can have: what the kernels declare themselves counts against 160 KiB too
+constexpr uint32_t kMaxLdsBytes = 160u * 1024u - kStepStaticLdsBytes;
 
 template <typename T>
 void upload(DeviceBuffer& b, const std::vector<T>& v) {
@@ -266,6 +267,7 @@ void World::compute_lds_layout() {
     L.u = take(4u * links, 4u);
     // the time-of-impact queries read the kinematics beside their colliders
     L.ccol = take(cfg_.ccd_mode == MR_CCD_HYBRID ? kColliderBytes * shapes : 0u, 4u);
+    L.swept = take(cfg_.ccd_mode == MR_CCD_HYBRID ? 4u * 2u * 64u : 0u, 4u);
     uint32_t union_end = off;
     off = union_start;
     L.col = take(kColliderBytes * shapes, 4u);
