@@ -813,8 +813,7 @@ int mr_mlp_adam_tensors(const MRMlpAdamTensorC* tensors, uint32_t tensor_count, 
         require(tensors != nullptr && tensor_count > 0u, "mr_mlp_adam: no tensors");
         for (uint32_t k = 0; k < tensor_count; ++k) {
             require(tensors[k].param && tensors[k].grad && tensors[k].m1 && tensors[k].m2, "mr_mlp_adam: null pointer");
-            require(tensors[k].count > 0u && tensors[k].count <= 0x7fffffffu && step >= 1u,
-                    "mr_mlp_adam: count and step must be positive");
+            require(tensors[k].count > 0u && step >= 1u, "mr_mlp_adam: count and step must be positive");
         }
         require(beta1 >= 0.0f && beta1 < 1.0f && beta2 >= 0.0f && beta2 < 1.0f && eps > 0.0f && lr >= 0.0f,
                 "mr_mlp_adam: hyper-parameters out of range");

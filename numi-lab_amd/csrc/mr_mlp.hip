@@ -443,7 +443,10 @@ __global__ void __launch_bounds__(1024) mlp_wgrad_kernel(uint32_t n, const float
 // One Adam step on up to kAdamTensors tensors: workgroup b works on the tensor
 // whose range of workgroups [first, next first) holds b. The network's six
 // parameters took six launches of a few microseconds each for 67,587 values.
+// A tensor of more than 2^31 values enters as several, and a launch stays below 2^32 threads.
 constexpr uint32_t kAdamTensors = 8u;
+constexpr uint32_t kAdamValues = 1u << 31;
+constexpr uint32_t kAdamGroups = 1u << 23;
 
 struct AdamArgs {
     MRMlpAdamTensorC tensor[kAdamTensors];
@@ -541,17 +544,33 @@ hipError_t mlp_adam(const MRMlpAdamTensorC* tensors, uint32_t tensor_count, floa
     }
     c1 = 1.0f - c1;
     c2 = 1.0f - c2;
-    for (uint32_t from = 0; from < tensor_count; from += kAdamTensors) {
-        AdamArgs args{};
-        uint32_t groups = 0u;
-        args.tensors = tensor_count - from < kAdamTensors ? tensor_count - from : kAdamTensors;
-        for (uint32_t k = 0; k < args.tensors; ++k) {
-            args.tensor[k] = tensors[from + k];
-            args.first[k] = groups;
-            groups += (args.tensor[k].count + 255u) / 256u;
+    AdamArgs args{};
+    uint32_t groups = 0u;
+    const auto launch = [&] {
+        if (groups > 0u)
+            hipLaunchKernelGGL(mr_mlp_adam_kernel, dim3(groups), dim3(256), 0, st, args, lr, beta1, beta2, eps, c1, c2);
+        args.tensors = 0u;
+        groups = 0u;
+    };
+    for (uint32_t k = 0; k < tensor_count; ++k) {
+        MRMlpAdamTensorC rest = tensors[k];
+        while (rest.count > 0u) {
+            const uint32_t n = rest.count < kAdamValues ? rest.count : kAdamValues;
+            const uint32_t own = (n + 255u) / 256u;
+            if (args.tensors == kAdamTensors || groups + own > kAdamGroups) launch();
+            args.tensor[args.tensors] = rest;
+            args.tensor[args.tensors].count = n;
+            args.first[args.tensors++] = groups;
+            groups += own;
+            rest.param += n;
+            rest.param_bf16 += rest.param_bf16 != nullptr ? n : 0u;
+            rest.grad += n;
+            rest.m1 += n;
+            rest.m2 += n;
+            rest.count -= n;
         }
-        hipLaunchKernelGGL(mr_mlp_adam_kernel, dim3(groups), dim3(256), 0, st, args, lr, beta1, beta2, eps, c1, c2);
     }
+    launch();
     return hipGetLastError();
 }
 

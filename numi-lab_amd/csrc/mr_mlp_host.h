@@ -16,7 +16,7 @@ hipError_t mlp_loss(const float* y_hat, const float* t, const float* out_scale, 
                     float* loss, float* scratch, hipStream_t st);
 hipError_t mlp_backward(const MRMlpWeightsC& w, const MRMlpTraceC& tr, const float* dy, uint32_t n, float* dz2,
                         float* dz1, const MRMlpGradsC& g, hipStream_t st);
-// One Adam step on every tensor, eight to a launch.
+// One Adam step on every tensor, up to eight to a launch.
 hipError_t mlp_adam(const MRMlpAdamTensorC* tensors, uint32_t tensor_count, float lr, float beta1, float beta2,
                     float eps, uint32_t step, hipStream_t st);
 

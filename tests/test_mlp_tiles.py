@@ -2,8 +2,8 @@
 restatement in oracle/mlp_oracle.py: one row, one short of a 16-row tile, a full
 tile and one more, a full 32-row chunk and one more, one more than the 16 x 32
 rows one pass of the weight-gradient waves covers and than the four passes they
-load at a time, and more 16-row tiles than the forward grid has workgroups; and
-the fused Adam launch against one launch per tensor.
+load at a time, and more 16-row tiles than the forward grid has workgroups; the
+fused Adam launch against one launch per tensor, and the largest tensors Adam takes.
 
 Tolerances as in test_mlp.py: gradients from the kernel's own trace within 2e-3
 of their scale (BF16 operands), activations within one BF16 rounding.
@@ -86,3 +86,42 @@ def test_adam_on_many_tensors_equals_one_at_a_time(gpu):
         assert torch.equal(half[0][k], half[1][k])
         assert all(torch.equal(u, v) for u, v in zip(one[k], many[k])), lengths[k]
         assert not torch.equal(many[k][0], base[k][0])
+
+
+@pytest.mark.parametrize("count", [2**31 - 1, 2**31, 2**31 + 1, 2**32 - 1])
+def test_adam_takes_every_count(count):
+    """A learning rate out of range is refused after the counts have been accepted; nothing is launched."""
+    from metalrobo import native as nat
+
+    b = nat.load()
+    p = ct.c_void_p(64)
+    with pytest.raises(nat.MetalRoboError, match="hyper-parameters"):
+        b.check(b.lib.mr_mlp_adam(p, None, p, p, p, count, -1.0, 0.9, 0.999, 1e-8, 1, None))
+    with pytest.raises(nat.MetalRoboError, match="count and step"):
+        b.check(b.lib.mr_mlp_adam(p, None, p, p, p, count, 1e-3, 0.9, 0.999, 1e-8, 0, None))
+
+
+@pytest.mark.gpu
+def test_adam_on_more_than_2_to_the_31_values(gpu):
+    """One tensor in two parts: values on both sides of the joint, and the last ones, as in a tensor of their own."""
+    import torch
+    from metalrobo import native as nat
+
+    n = 2**31 + 300
+    if torch.cuda.mem_get_info()[0] < 6 * 4 * n:
+        pytest.skip("needs 52 GB of device memory")
+    b = nat.load()
+    at = torch.tensor([0, 255, 256, 2**31 - 1, 2**31, 2**31 + 255, 2**31 + 256, n - 1], device="cuda")
+    gen = torch.Generator().manual_seed(4)
+    small = [torch.rand(len(at), generator=gen).cuda() for _ in range(4)]
+    half = [torch.zeros(k, dtype=torch.bfloat16, device="cuda") for k in (len(at), n)]
+    large = [torch.zeros(n, device="cuda") for _ in range(4)]
+    for u, v in zip(large, small):
+        u[at] = v
+    p = lambda v: ct.c_void_p(v.data_ptr())  # noqa: E731
+    print("adam on", n, "values", flush=True)
+    for (w, g, m1, m2), h in ((small, half[0]), (large, half[1])):
+        b.check(b.lib.mr_mlp_adam(p(w), p(h), p(g), p(m1), p(m2), w.numel(), 1e-3, 0.9, 0.999, 1e-8, 2, None))
+    torch.cuda.synchronize()
+    assert torch.equal(half[1][at], half[0]) and half[0].count_nonzero() == len(at)
+    assert all(torch.equal(u[at], v) for u, v in zip(large, small))
