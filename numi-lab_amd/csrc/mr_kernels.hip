@@ -4863,13 +4863,9 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
                     uint32_t my_fail = MR_INVALID_INDEX;
                     for (uint32_t l = 0; l < levels; ++l) {
                         const uint32_t first = pk & 0xffffu, end = pk_next & 0xffffu, art_c = pk >> 16;
-                        const uint32_t c0 = cc;
-                        const HotConstraint h0 = rec;
                         const uint32_t ln = l + 1u < levels ? l + 1u : 0u;
                         pk = level_pack(ln);
                         pk_next = level_pack(ln + 1u);
-                        cc = sched_contact(pk & 0xffffu, (pk_next & 0xffffu) - (pk & 0xffffu));
-                        rec = e.hot[cc];
                         auto scene_contact = [&](uint32_t c, const HotConstraint& hk) {
                             const bool da = (hk.kind & mr::kHotDynamicA) != 0u, db = (hk.kind & mr::kHotDynamicB) != 0u;
                             float4* sa = e.sbody + (da ? hk.body_a - nl : 0u) * kSolverBodyVectors;
@@ -4895,12 +4891,22 @@ __device__ __forceinline__ void control_step(const KernelArgs& args, uint32_t en
                             e.lam[3u * c + 1u] = cand[1];
                             e.lam[3u * c + 2u] = cand[2];
                         };
-                        if (first + lane < end) scene_contact(c0, h0);
-                        for (uint32_t p = first + kLanes + lane; p < end; p += kLanes) {
-                            const uint32_t c = e.sord[p];
-                            scene_contact(c, e.hot[c]);
+                        // Most levels of a robot beside a few objects hold its own
+                        // contact only, and fetch no record. (With one fetched for
+                        // every level, 512 chains of 20 links and a free box, 2
+                        // control steps to residual 1e-5, took 40.1 ms, now 35.1.)
+                        if (first < end || (pk & 0xffffu) < (pk_next & 0xffffu)) {
+                            const uint32_t c0 = cc;
+                            const HotConstraint h0 = rec;
+                            cc = sched_contact(pk & 0xffffu, (pk_next & 0xffffu) - (pk & 0xffffu));
+                            rec = e.hot[cc];
+                            if (first + lane < end) scene_contact(c0, h0);
+                            for (uint32_t p = first + kLanes + lane; p < end; p += kLanes) {
+                                const uint32_t c = e.sord[p];
+                                scene_contact(c, e.hot[c]);
+                            }
+                            __builtin_amdgcn_wave_barrier();
                         }
-                        __builtin_amdgcn_wave_barrier();
                         if (art_c != 0u) {
                             k_art = k_art + 1u < nart ? k_art + 1u : 0u;
                             cn = art_at(k_art);

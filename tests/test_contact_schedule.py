@@ -1,6 +1,6 @@
 """The level schedule of the ordered sweeps against the oracle's plain index order, bit for bit, where
 the schedule can go wrong: more than 64 levels (one slab under many boxes), more than 64 contacts
-in few levels, an articulation touching dynamic bodies, and updates that are not finite (the first
+in few levels, an articulation touching dynamic bodies, one beside a dynamic body, and updates that are not finite (the first
 failing contact in index order is reported)."""
 
 import numpy as np
@@ -30,6 +30,21 @@ def world(movers, links=(), dofs=(), link_shapes=(), nq=0, envs=2):
     bodies.append(mu.body(0.0, [1, 1, 1], motion=0))
     shapes.append(mu.shape(len(bodies) - 1, PLANE, [], rot=mu.Y_TO_Z))
     return mu.CustomWorld(bodies, list(dofs), shapes, link_count=nl, root_type=0, nq=nq, nv=nq, envs=envs)
+
+
+def beside(rng):
+    """A chain of 20 box links lying on the plane and one free box apart: 80 levels of an articulated
+    contact each, of which only the first four hold a contact between scene bodies too."""
+    links, dofs, shapes = [mu.body(1.0, [0.01] * 3)], [], []
+    for i in range(1, 21):
+        links.append(mu.body(1.5, [0.02, 0.004, 0.02], parent=i - 1, joint_type=0, q_index=i - 1, v_index=i - 1,
+                             axis=(0, 0, 1), parent_anchor=(0, 0.12, 0) if i > 1 else (0, 0, 0.0495),
+                             child_anchor=(0, -0.12, 0)))
+        dofs.append(mu.dof(i, i - 1))
+        shapes.append(mu.shape(i, BOX, [0.1, 0.1, 0.05]))
+    movers = [((0.06, 0.06, 0.06), 0.8)]
+    w = world(movers, links, dofs, shapes, nq=20)
+    return w, state_of(w, [(2.0, 0.0, 0.0595)], [0.8], rng), 20
 
 
 def state_of(w, positions, masses, rng, speed=0.3):
@@ -109,7 +124,7 @@ def compare(w, scene, nq, steps=6, expect_failure=False, fails_at=None, **cfg_ar
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("tolerance", [0.0, 1.0e-5])
-@pytest.mark.parametrize("scene,least", [(slab, 80), (grid, 65), (linked, 20)])
+@pytest.mark.parametrize("scene,least", [(slab, 80), (grid, 65), (linked, 20), (beside, 84)])
 def test_scheduled_sweeps_match_the_index_order(gpu, scene, least, tolerance):
     w, states, nq = scene(np.random.default_rng(4))
     assert compare(w, states, nq, residual_tolerance=tolerance) >= least
