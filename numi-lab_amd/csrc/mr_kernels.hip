@@ -3141,8 +3141,9 @@ MRD_INL float rel_row(uint32_t kind, V3 d, V3 va, V3 vb, float art_dot) {
 // is one more than the largest level of the earlier contacts at its nodes; the
 // contacts of a level share no node, so those between scene bodies run one per
 // lane, and the at most one articulated contact of a level runs on the whole wave
-// (its dot products are folds over the DoF lanes). A pile of 20 boxes has about
-// 58 contacts (2.5 of them articulated) in 7 levels. An update is a serial chain of
+// (its dot products are folds over the DoF lanes). A pile of 20 boxes still
+// landing has about 58 contacts (2.5 of them articulated) in 7 levels, a settled
+// one 93. An update is a serial chain of
 // LDS reads and about 250 instructions whatever the number of active lanes, so the
 // levels, not the contacts, set the sweep's time. Measured, 2 control steps: 1024
 // chain-and-boxes worlds 6.00 -> 2.90 ms, 1500 random trees 13.2 -> 5.95 ms, 300
